@@ -121,3 +121,29 @@ def test_score_error_is_that_of_samples_taken_one_by_one(ctx, n, radius):
     rms = lambda v: np.sqrt(np.mean(v ** 2))  # noqa: E731
     print(f"score error: refinement {rms(cc - exact):.2e}, adjoint entry {rms(ref - exact):.2e}")
     assert rms(cc - exact) < 1.25 * rms(ref - exact)
+
+
+@pytest.mark.parametrize("n,radius,table", [(8, 3.9, "c64"), (16, 7.9, "f16"), (33, 16.4, "c64"), (64, 31.9, "c64"),
+                                            (75, 37.4, "f16"), (128, 63.7, "c64")])
+def test_samples_at_the_tables_edge(ctx, n, radius, table):
+    """Supports past (n - 1) / 2 reach the table's last plane on every axis: white
+    particles whose spectra are zero but in that last shell, so that one wrong texel
+    of its ~100 n samples shows."""
+    al, R, s = _aligner(n, 12, radius, table, n)
+    rng = np.random.default_rng(n)
+    ref = rng.standard_normal((n, n, n)).astype(np.float32)
+    al = BatchAligner(n, ref, np.ones((n, n, n), np.float32), support_radius=radius, table=table,
+                      tuning={"params": {table: {str(n): {"grad_kernel": 0}}}})
+    al.set_particles([rng.standard_normal((n, n, n)).astype(np.float32) for _ in R], [None] * len(R),
+                     [np.eye(3)] * len(R))
+    a = np.fft.fftfreq(n) * n
+    kz, kx, ky = np.meshgrid(a, np.arange(n // 2 + 1.0), a, indexing="ij")
+    shell = (kx ** 2 + ky ** 2 + kz ** 2 > ((n - 1) / 2) ** 2).ravel()
+    al.Q = DeviceArray.from_numpy(np.where(shell, al.Q.get(), 0).astype(np.complex64), ctx=al.ctx)
+    al.N = DeviceArray.from_numpy(np.where(shell, al.N.get(), 0).astype(np.float32), ctx=al.ctx)
+    cc, ref_cc = _scores(al, R, s)
+    assert np.max(np.abs(cc - ref_cc)) <= 2e-6 * max(1.0, np.max(np.abs(ref_cc)))
+    Rd, sd, _ = al.refine(R, s, iters=1)
+    Rh, sh, _ = _host_refine(al, R, s, iters=1)
+    same = (np.max(np.abs(Rd - R), axis=(1, 2)) > 0) == (np.max(np.abs(Rh - R), axis=(1, 2)) > 0)
+    assert np.max(np.abs(Rd - Rh)[same], initial=0.0) < 2e-5 and np.max(np.abs(sd - sh)[same], initial=0.0) < 3e-4
