@@ -74,7 +74,8 @@ def _scores(al, R, s):
     (33, 17, 15.9, "c64"),     # odd box, one particle past a workgroup's waves
     (64, 70, 14.0, "c64"),     # several runs of particles per brick
     (75, 5, 28.7, "f16"),
-    (128, 2, 63.5, "c64"),     # the most cubes and bricks
+    (128, 2, 63.5, "c64"),     # 9,405 cubes in 2,160 bricks
+    (128, 2, 63.99, "c64"),    # the most of both: 9,598 in 2,316
 ])
 def test_steps_match_the_adjoint_entry(ctx, n, count, radius, table):
     al, R, s = _aligner(n, count, radius, table, n)
