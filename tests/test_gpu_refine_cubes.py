@@ -8,7 +8,7 @@ import pytest
 
 from emclarity_amd import _lib
 from emclarity_amd.batched import BatchAligner
-from emclarity_amd.device import DeviceArray
+from emclarity_amd.device import Context, DeviceArray
 from emclarity_amd.workload import random_rotation
 
 from test_gpu_batched import _host_refine
@@ -148,3 +148,20 @@ def test_samples_at_the_tables_edge(ctx, n, radius, table):
     Rh, sh, _ = _host_refine(al, R, s, iters=1)
     same = (np.max(np.abs(Rd - R), axis=(1, 2)) > 0) == (np.max(np.abs(Rh - R), axis=(1, 2)) > 0)
     assert np.max(np.abs(Rd - Rh)[same], initial=0.0) < 2e-5 and np.max(np.abs(sd - sh)[same], initial=0.0) < 3e-4
+
+
+def test_supports_that_print_alike_are_kept_apart(ctx):
+    """4.9999999 and 5.0 differ by the frequencies at |k| = 5, some of them in cubes
+    of their own: the call with the larger may not meet the smaller's cubes."""
+    cc = []
+    for before in (None, 4.9999999):
+        al, R, s = _aligner(16, 4, 5.0, "c64", 1)
+        own = Context(0)
+        al.ctx = own
+        al.ctx.wait_for(ctx)
+        args = lambda: (DeviceArray.from_numpy(np.ascontiguousarray(R.reshape(-1, 9)), ctx=own),  # noqa: E731
+                        DeviceArray.from_numpy(s.copy(), ctx=own))
+        if before:
+            al.refine_device(*args(), iters=0, support_radius=before).get()
+        cc.append(al.refine_device(*args(), iters=0).get())
+    np.testing.assert_array_equal(cc[0], cc[1])
