@@ -165,3 +165,22 @@ def test_supports_that_print_alike_are_kept_apart(ctx):
             al.refine_device(*args(), iters=0, support_radius=before).get()
         cc.append(al.refine_device(*args(), iters=0).get())
     np.testing.assert_array_equal(cc[0], cc[1])
+
+
+@pytest.mark.parametrize("table", ["c64", "f16"])
+def test_steps_from_poses_that_are_not_rotations(ctx, table):
+    """Stretched, sheared and singular start matrices (a projection maps the table
+    onto a plane): the shift's gradient sums k itself, as no inverse gives it back."""
+    al, R, s = _aligner(36, 6, 12.3, table, 4)
+    R[1] *= 1.3
+    R[2] = R[2] @ np.array([[1.0, 0.6, 0], [0, 1, 0], [0, 0, 1]])
+    R[3] = R[3] @ np.diag([1.0, 1.0, 0.0])
+    R[4] = np.outer(R[4][:, 0], R[4][0])
+    R[5] *= 1.0001                                # within the bricks' halo: staged
+    Rd, sd, cd = al.refine(R, s, iters=1)
+    Rh, sh, ch = _host_refine(al, R, s, iters=1)
+    assert np.max(np.abs(cd - ch)) <= 2e-6
+    # as above; both forms decide alike on all but ties
+    same = (np.max(np.abs(Rd - R), axis=(1, 2)) > 0) == (np.max(np.abs(Rh - R), axis=(1, 2)) > 0)
+    assert same.sum() >= 5 and np.max(np.abs(sd - s)[3:5]) > 0
+    assert np.max(np.abs(Rd - Rh)[same]) < 4e-5 and np.max(np.abs(sd - sh)[same]) < 3e-4
