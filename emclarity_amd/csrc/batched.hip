@@ -506,7 +506,7 @@ __global__ void __launch_bounds__(kBatchThreads) __attribute__((amdgpu_waves_per
 // operand B (4 x 16) of
 //   y: G[dy][dz]  = sum_ky e^{2 pi i ky dy / n} T[ky][dz]   (16 a strip)
 // and lane l then holds G[4 (l / 16) + i][l % 16] for
-//   x: map[dx][dy][dz] += m Re(G e^{2 pi i kx dx / n})   (m = 2, 1 at kx = 0)
+//   x: map[dx][dy][dz] += m Re(G e^{2 pi i kx dx / n})   (m = 1 at kx = 0 and n / 2 = kx, else 2)
 // on 4 D registers that stay with the wave for its whole group. Nothing goes
 // through LDS but the twiddles, and no barrier follows their staging.
 // A group of strips writes its unit's partial map in register order,
@@ -565,7 +565,7 @@ __global__ void __launch_bounds__(kStripSlots* kWave) __attribute__((amdgpu_wave
     const int yy = ky < 0 ? ky + n : (ky >= n ? ky - n : ky);
     const float fkx = (float)kx, fky = (float)ky;
     const float bx = m00 * fkx + m01 * fky, by = m10 * fkx + m11 * fky, bz = m20 * fkx + m21 * fky;
-    // the support ends at n/2 - 1 on each axis (an odd box has a frequency past it)
+    // the support ends at n/2 - 1 along y and z (an odd box has a frequency past it)
     const float k2 = abs(ky) < n / 2 ? (float)(kx * kx + ky * ky) : kmax2 + 1.0f;
     floatx4 tr = {0.0f, 0.0f, 0.0f, 0.0f}, ti = {0.0f, 0.0f, 0.0f, 0.0f};
     float dpart = 0.0f;
@@ -607,7 +607,7 @@ __global__ void __launch_bounds__(kStripSlots* kWave) __attribute__((amdgpu_wave
       step(va, ta, qa, wa, za);
       if (z0 + 4 <= st.z) step(vb, tb, qb, wb, zb < n ? zb : 0);  // uniform
     }
-    const float mk = kx == 0 ? 1.0f : 2.0f;  // the support stays below the Nyquist plane
+    const float mk = kx == 0 || (n % 2 == 0 && kx == n / 2) ? 1.0f : 2.0f;
     norm += (double)(mk * dpart);
     const floatx4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
     floatx4 g0 = zero, g1 = zero, g2 = zero, g3 = zero;
@@ -1250,7 +1250,7 @@ static StripSet strip_set(emc_ctx* ctx, int n, float kmax2, int want) {
     return r;
   }
   std::vector<int4> strips;
-  for (int kx = 0; kx <= n / 2 - 1 && (float)(kx * kx) <= kmax2; ++kx) {
+  for (int kx = 0; kx <= n / 2 && (float)(kx * kx) <= kmax2; ++kx) {  // the columns of support_schedule
     int w = 0;
     while (w + 1 <= n / 2 - 1 && (float)(kx * kx + (w + 1) * (w + 1)) <= kmax2) ++w;
     for (int y0 = -w; y0 <= w; y0 += 16) {

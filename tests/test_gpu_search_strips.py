@@ -1,7 +1,7 @@
-"""The search's matrix-core form against the column passes: the same particles
-scored in one call of many units (strips) and one particle at a time (passes:
-fewer than 2,048 units), at boxes whose last ky tile, kz step and table region
-differ; both against each other to FP32 summation order."""
+"""The search's matrix-core form against the column passes (the same particles
+scored in one call of many units, which takes the strips, and one particle at a
+time, under 2,048 units, which takes the passes) at boxes whose last ky tile, kz
+step and table region differ, to FP32 summation order."""
 import numpy as np
 import pytest
 
@@ -23,9 +23,23 @@ def test_strips_match_passes(ctx, n, radius, peak_radius, table):
     ref = np.exp(-((x - 0.1 * n) ** 2 + y ** 2 + 2 * z ** 2) / (2 * (0.12 * n) ** 2))
     ref += 0.6 * np.exp(-((x + 0.2 * n) ** 2 + (y - 0.1 * n) ** 2 + z ** 2) / (2 * (0.05 * n) ** 2))
     grid = eulerSearch("C1", 15, 5, 15, 5)
-    P = -(-2048 // len(grid)) + 1
     parts = [(np.roll(ref, tuple(rng.integers(-2, 3, 3)), (0, 1, 2)) + 0.2 * rng.standard_normal((n, n, n)))
-             .astype(np.float32) for _ in range(P)]
+             .astype(np.float32) for _ in range(-(-2048 // len(grid)) + 1)]
+    _compare(n, radius, peak_radius, table, rng, grid, ref, parts)
+
+
+@pytest.mark.parametrize("n,radius,peak_radius,table", [(9, 4.4, 4, "c64"), (31, 15.4, 6, "c64"), (41, 20.4, 4, "f16")])
+def test_odd_boxes_keep_their_last_x_plane(ctx, n, radius, peak_radius, table):
+    """An odd box has a plane kx = (n - 1) / 2 inside supports past it (white volumes)."""
+    rng = np.random.default_rng(n)
+    ref = rng.standard_normal((n, n, n))
+    grid = eulerSearch("C1", 15, 5, 15, 5)
+    parts = [rng.standard_normal((n, n, n)).astype(np.float32) for _ in range(-(-2048 // len(grid)))]
+    _compare(n, radius, peak_radius, table, rng, grid, ref, parts)
+
+
+def _compare(n, radius, peak_radius, table, rng, grid, ref, parts):
+    P = len(parts)
     starts = [random_rotation(rng) for _ in range(P)]
     al = BatchAligner(n, ref.astype(np.float32), np.ones((n, n, n), np.float32), support_radius=radius,
                       peak_radius=peak_radius, table=table)
