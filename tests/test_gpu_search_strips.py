@@ -1,13 +1,15 @@
 """The search's matrix-core form against the column passes (the same particles
 scored in one call of many units, which takes the strips, and one particle at a
 time, under 2,048 units, which takes the passes) at boxes whose last ky tile, kz
-step and table region differ, to FP32 summation order."""
+step and table region differ, to FP32 summation order; and against the FP64 oracle."""
 import numpy as np
 import pytest
 
+from emclarity_amd import synthetic as S
 from emclarity_amd.batched import BatchAligner
 from emclarity_amd.geometry import eulerSearch
-from emclarity_amd.workload import random_rotation
+from emclarity_amd.workload import local_matrix, random_rotation
+from oracle import emc_oracle as O
 
 pytestmark = pytest.mark.gpu
 
@@ -54,3 +56,27 @@ def _compare(n, radius, peak_radius, table, rng, grid, ref, parts):
         assert np.max(np.abs(score[i] - s1[0])) < 1e-5 * np.max(np.abs(s1))
         # the peak's parabola; a tie of two voxels may fall to either
         assert np.mean(np.max(np.abs(shift[i] - d1[0]), axis=1) < 1e-3) > 0.99
+
+
+@pytest.mark.parametrize("table", ["c64", "f16"])
+def test_strips_match_the_oracle(ctx, table):
+    """One particle from 128 start orientations over 16 grid points: 2,048 units, every
+    85th against the full-grid FP64 restatement, to the bounds of the passes' test."""
+    n, P = 32, 128
+    bp = O.bandpass3d((n, n, n), 1e-3, 40.0, 8.0, 2.5)
+    truth = (40.0, 30.0, 20.0)
+    c = S.make_align_case(11, n=n, euler=truth, snr=1.0, n_blobs=16, blob_radius=0.22 * n)
+    rng = np.random.default_rng(2)
+    starts = [np.eye(3) if i % 2 else local_matrix(*rng.uniform(-20, 20, 3)) for i in range(P)]
+    al = BatchAligner(n, c.ref, bp.astype(np.float32), peak_radius=6, table=table)
+    al.set_particles([c.particle] * P, [None] * P, starts)
+    pts = np.array([truth] + [tuple(rng.uniform(0, 180, 3)) for _ in range(15)])
+    score, shift = al.search(pts)
+    assert score.size >= 2048
+    F2 = O.batch_reference_spectrum(c.ref, table)
+    bpp = O.batch_prepare(c.particle, bp, np.ones((n, n, n), np.float32), al.support)
+    for unit in range(0, P * len(pts), 85):
+        i, k = divmod(unit, len(pts))
+        sc, sh = O.batch_score_map(F2, n, bpp, starts[i] @ local_matrix(*pts[k]), 6)
+        assert abs(score[i, k] - sc) < 1e-4 * abs(sc), (i, k, score[i, k], sc)
+        assert np.max(np.abs(shift[i, k] - sh)) < 2e-3, (i, k, shift[i, k], sh)
