@@ -3,6 +3,8 @@ entry (emc_align_eval_grad, support-list order): scores and the steps taken
 from the gradients, at the smallest and largest supports, odd boxes, both
 table formats, few and many particles, and poses that are not rotations
 (gathered from the table instead of the staged bricks)."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -184,3 +186,39 @@ def test_steps_from_poses_that_are_not_rotations(ctx, table):
     same = (np.max(np.abs(Rd - R), axis=(1, 2)) > 0) == (np.max(np.abs(Rh - R), axis=(1, 2)) > 0)
     assert same.sum() >= 5 and np.max(np.abs(sd - s)[3:5]) > 0
     assert np.max(np.abs(Rd - Rh)[same]) < 4e-5 and np.max(np.abs(sd - sh)[same]) < 3e-4
+
+
+def test_runs_of_particles_within_the_scratch_bound(ctx):
+    """200 particles of 128^3 over their whole support take two runs within 1 GiB of
+    scratch: as many bytes as that, and the poses of the particles refined by themselves."""
+    n, count = 128, 200
+    al, R, s = _aligner(n, 2, 62.9, "c64", 3)
+    rng = np.random.default_rng(1)
+    own = Context(0)
+    own.wait_for(ctx)
+    al.ctx, al.n_part = own, count
+    for name in ("Q", "N", "A"):
+        a = getattr(al, name).get()
+        setattr(al, name, DeviceArray.from_numpy(np.ascontiguousarray(np.tile(a, (count // 2,) + (1,) * (a.ndim - 1))),
+                                                 ctx=own))
+    R = R[np.arange(count) % 2]
+    s = rng.uniform(-2.0, 2.0, (count, 3))
+    dev = lambda v: DeviceArray.from_numpy(np.ascontiguousarray(v), ctx=own)  # noqa: E731
+    Rd, sd = dev(R.reshape(-1, 9)), dev(s)
+    own.synchronize()
+
+    def free():
+        f, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert _lib.load().hipMemGetInfo(ctypes.byref(f), ctypes.byref(total)) == 0
+        return f.value
+    before = free()
+    cc = al.refine_device(Rd, sd, iters=2).get()
+    assert before - free() < 1.1 * 2 ** 30
+    al.n_part = 4
+    for p0 in (0, 98, 196):
+        q = slice(p0, p0 + 4)
+        R4, s4 = dev(R[q].reshape(-1, 9)), dev(s[q])
+        c4 = al.refine_device(R4, s4, iters=2).get()   # particles repeat with period 2
+        np.testing.assert_array_equal(c4, cc[q])
+        np.testing.assert_array_equal(R4.get(), Rd.get()[q])
+        np.testing.assert_array_equal(s4.get(), sd.get()[q])
