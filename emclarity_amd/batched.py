@@ -245,6 +245,16 @@ def support_voxels(n, support):
     return int(np.count_nonzero(r2 <= support * support))
 
 
+def search_uses_strips(support, table, peak_radius, units):
+    """Whether emc_align_batched scores `units` (particle, orientation) pairs
+    over `support` by strips on the matrix cores (restated from its dispatch:
+    at least 2,048 units, and the entries of the half ball |j| <= 2 r + 1 in
+    2.5 MB) instead of the column passes."""
+    entry = 4 * (8 if table == "c64" else 4)
+    region = 2 / 3 * math.pi * (2 * math.sqrt(np.float32(support * support)) + 1) ** 3 * entry
+    return peak_radius in (4, 6) and units >= 2048 and region <= 2.5e6
+
+
 def fused_schedule(n, support, tile=16, width=256):
     """Column schedule of the fused search kernel (restated from its host
     builder): columns (kx, ky, h) of the half disk kx^2 + ky^2 <= r^2, tiled
