@@ -77,7 +77,9 @@ def _scores(al, R, s):
     (64, 70, 14.0, "c64"),     # several runs of particles per brick
     (75, 5, 28.7, "f16"),
     (128, 2, 63.5, "c64"),     # 9,405 cubes in 2,160 bricks
-    (128, 2, 63.99, "c64"),    # the most of both: 9,598 in 2,316
+    (128, 5, 63.99, "c64"),    # the most of both: 9,598 in 2,316
+    (8, 5, 3.4, "f16"),        # the fewest particles whose bricks are staged, the most that are gathered
+    (75, 4, 36.0, "c64"),
 ])
 def test_steps_match_the_adjoint_entry(ctx, n, count, radius, table):
     al, R, s = _aligner(n, count, radius, table, n)
@@ -169,22 +171,21 @@ def test_supports_that_print_alike_are_kept_apart(ctx):
     np.testing.assert_array_equal(cc[0], cc[1])
 
 
-@pytest.mark.parametrize("table", ["c64", "f16"])
-def test_steps_from_poses_that_are_not_rotations(ctx, table):
+@pytest.mark.parametrize("table,count", [("c64", 6), ("f16", 6), ("c64", 4)])
+def test_steps_from_poses_that_are_not_rotations(ctx, table, count):
     """Stretched, sheared and singular start matrices (a projection maps the table
     onto a plane): the shift's gradient sums k itself, as no inverse gives it back."""
-    al, R, s = _aligner(36, 6, 12.3, table, 4)
-    R[1] *= 1.3
-    R[2] = R[2] @ np.array([[1.0, 0.6, 0], [0, 1, 0], [0, 0, 1]])
-    R[3] = R[3] @ np.diag([1.0, 1.0, 0.0])
-    R[4] = np.outer(R[4][:, 0], R[4][0])
-    R[5] *= 1.0001                                # within the bricks' halo: staged
+    al, R, s = _aligner(36, count, 12.3, table, 4)
+    change = [lambda A: A, lambda A: 1.3 * A, lambda A: A @ np.array([[1.0, 0.6, 0], [0, 1, 0], [0, 0, 1]]),
+              lambda A: A @ np.diag([1.0, 1.0, 0.0]), lambda A: np.outer(A[:, 0], A[0]),
+              lambda A: 1.0001 * A]             # the last within the bricks' halo: staged
+    R = np.stack([f(A) for f, A in zip(change[-count:], R)])
     Rd, sd, cd = al.refine(R, s, iters=1)
     Rh, sh, ch = _host_refine(al, R, s, iters=1)
     assert np.max(np.abs(cd - ch)) <= 2e-6
     # as above; both forms decide alike on all but ties
     same = (np.max(np.abs(Rd - R), axis=(1, 2)) > 0) == (np.max(np.abs(Rh - R), axis=(1, 2)) > 0)
-    assert same.sum() >= 5 and np.max(np.abs(sd - s)[3:5]) > 0
+    assert same.sum() >= count - 1 and np.max(np.abs(sd - s)[-3:-1]) > 0
     assert np.max(np.abs(Rd - Rh)[same]) < 4e-5 and np.max(np.abs(sd - sh)[same]) < 3e-4
 
 
@@ -214,11 +215,11 @@ def test_runs_of_particles_within_the_scratch_bound(ctx):
     before = free()
     cc = al.refine_device(Rd, sd, iters=2).get()
     assert before - free() < 1.1 * 2 ** 30
-    al.n_part = 4
-    for p0 in (0, 98, 196):
-        q = slice(p0, p0 + 4)
-        R4, s4 = dev(R[q].reshape(-1, 9)), dev(s[q])
-        c4 = al.refine_device(R4, s4, iters=2).get()   # particles repeat with period 2
-        np.testing.assert_array_equal(c4, cc[q])
-        np.testing.assert_array_equal(R4.get(), Rd.get()[q])
-        np.testing.assert_array_equal(s4.get(), sd.get()[q])
+    al.n_part = 8
+    for p0 in (0, 96, 192):
+        q = slice(p0, p0 + 8)
+        R8, s8 = dev(R[q].reshape(-1, 9)), dev(s[q])
+        c8 = al.refine_device(R8, s8, iters=2).get()   # particles repeat with period 2
+        np.testing.assert_array_equal(c8, cc[q])
+        np.testing.assert_array_equal(R8.get(), Rd.get()[q])
+        np.testing.assert_array_equal(s8.get(), sd.get()[q])
