@@ -1228,8 +1228,8 @@ const int* support_schedule(emc_ctx* ctx, int n, float kmax2, int* ngroups) {
   return d;
 }
 
-// Strips of the support ball (align_strip_kernel), cached per (n, radius,
-// groups) in the context: int4 {kx, first ky, largest |kz|, last of its kx}, and the starts
+// Strips of the support ball (align_strip_kernel), cached per (n, largest k^2
+// inside, groups) in the context: int4 {kx, first ky, largest |kz|, last of its kx}, and the starts
 // of `want` groups of consecutive strips of about equal work.
 struct StripSet {
   const int4* strips;
@@ -1239,7 +1239,7 @@ struct StripSet {
 
 static StripSet strip_set(emc_ctx* ctx, int n, float kmax2, int want) {
   char key[96];
-  snprintf(key, sizeof(key), "strips_%d_%.6f_g%d", n, (double)kmax2, want);
+  snprintf(key, sizeof(key), "strips_%d_%d_g%d", n, (int)kmax2, want);
   StripSet r{};
   auto it = ctx->scratch.find(key);
   auto mt = ctx->meta.find(key), ms = ctx->meta.find(std::string(key) + "_s");

@@ -7,6 +7,7 @@ import pytest
 
 from emclarity_amd import synthetic as S
 from emclarity_amd.batched import BatchAligner
+from emclarity_amd.device import Context
 from emclarity_amd.geometry import eulerSearch
 from emclarity_amd.workload import local_matrix, random_rotation
 from oracle import emc_oracle as O
@@ -56,6 +57,25 @@ def _compare(n, radius, peak_radius, table, rng, grid, ref, parts):
         assert np.max(np.abs(score[i] - s1[0])) < 1e-5 * np.max(np.abs(s1))
         # the peak's parabola; a tie of two voxels may fall to either
         assert np.mean(np.max(np.abs(shift[i] - d1[0]), axis=1) < 1e-3) > 0.99
+
+
+def test_radii_that_print_alike_are_kept_apart(ctx):
+    """radius^2 = 3.9999998 and 4.0 print the same and differ by the frequencies at |k| = 2."""
+    rng = np.random.default_rng(1)
+    n, P, grid = 8, 147, eulerSearch("C1", 15, 10, 15, 10)[:14]
+    vol = rng.standard_normal((n, n, n)).astype(np.float32)
+    part = rng.standard_normal((n, n, n)).astype(np.float32)
+    starts = [random_rotation(rng) for _ in range(P)]
+    score = []
+    for before in (None, float(np.sqrt(3.9999998))):
+        own = Context(0)
+        al = BatchAligner(n, vol, np.ones((n, n, n), np.float32), support_radius=2.0, peak_radius=4, ctx=own)
+        al.set_particles([part] * P, [None] * P, starts)
+        if before:
+            al.search(grid, before)
+        score.append(al.search(grid, 2.0)[0])
+    assert score[0].size >= 2048
+    np.testing.assert_array_equal(score[0], score[1])
 
 
 @pytest.mark.parametrize("table", ["c64", "f16"])
