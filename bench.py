@@ -302,7 +302,7 @@ def search_kernel(step, kt, steps):
         flops += fused_flops_per_unit(n, r, 6) * u
         samples += fused_samples_per_unit(n, r) * u
     sec = k["_ms"] * 1e-3
-    return {"kernel": "align_strip_kernel<6> / align_pass_kernel<6>", "avg_us": k["avg_us"], "launches": k["_n"],
+    return {"kernel": "align_pass_kernel<6>", "avg_us": k["avg_us"], "launches": k["_n"],
             "achieved_tflops": round(flops * steps / sec / 1e12, 3),
             "frac_fp32_peak": round(flops * steps / sec / 1e12 / FP32_PEAK_TFLOPS, 4),
             "gsamples_per_s": round(samples * steps / sec / 1e9, 2)}

@@ -1330,9 +1330,9 @@ void launch_search(emc_ctx* ctx, int peak_radius, const void* F2, int n, const f
   // and the units fill the device with a wave each; else the column passes,
   // which keep resident units on one patch of the table. Measured, 28
   // orientations, 0.6 x the support unless noted (strips against passes):
-  // 800 x 64^3 1.53 / 1.98 ms (1.8 MB), fp16 table 1.39 / 1.93, 1,000 x 48^3
-  // 1.10 / 1.20, 400 x 40^3 full support 0.87 / 1.07 (2.2 MB), 100 x 64^3 0.24 /
-  // 0.29; the other way 300 x 80^3 1.46 / 1.33 (3.8 MB), 300 x 96^3 2.75 / 2.25,
+  // 800 x 64^3 1.53 / 1.98 ms (2.1 MB), fp16 table 1.39 / 1.93, 1,000 x 48^3
+  // 1.10 / 1.20, 400 x 40^3 full support 0.87 / 1.07 (2.4 MB), 100 x 64^3 0.24 /
+  // 0.29; the other way 300 x 80^3 1.46 / 1.33 (3.9 MB), 300 x 96^3 2.75 / 2.25,
   // 20 x 64^3 (560 units) 0.13 / 0.11.
   const double R = 2.0 * std::sqrt((double)kmax2) + 1.0;
   const double region = 2.0 / 3.0 * M_PI * R * R * R * 4 * sizeof(typename Tab::T);

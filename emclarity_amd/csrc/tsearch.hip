@@ -461,10 +461,12 @@ emc_status emc_template_search_chunk(emc_ctx* ctx, const float* d_chunk, const i
     // 0 selects the padded-volume R2C instead)
     const int pmode = tune_value(ctx, "tsearch_pruned", 0, 2);
     const bool pruned = pmode != 0 && td[0] <= kTMax && td[1] <= kTMax && td[2] <= kTMax;
-    // The valid area's own inverse wherever the chunk's edges allow it (factors
-    // 2, 3 and 5, up to ~850 voxels: chunks are cut so). 24 orientations of a
-    // 48^3 template over 360 x 384 x 324: 9.6 ms against 20.1 ms with the library's
-    // inverse of the whole chunk; longer edges do not fit a tile of 8 columns in LDS.
+    // The valid area's own inverse wherever the chunk's edges allow it: factors 2,
+    // 3 and 5, and up to 903 voxels along y and z, 1,476 along x, as longer columns do
+    // not fit a tile of 8 in LDS. Most edges that chunks are cut to are such; those
+    // with a factor 7 (168, 224, 336, 756, 896, 1008) and 960 to 1,024 along y or z take
+    // the library's inverse of the whole chunk. 24 orientations of a 48^3 template
+    // over 360 x 384 x 324: 9.6 ms against 20.1 ms with the library's.
     const bool columns = pruned && pmode == 2 && ts_inverse_supported(cd);
     emc_fft_plan* plan1 = cached_plan(ctx, cd[0], cd[1], cd[2], 1);
     emc_fft_plan* planb = columns ? nullptr : cached_plan(ctx, cd[0], cd[1], cd[2], blk);

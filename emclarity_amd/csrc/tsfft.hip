@@ -5,7 +5,7 @@
 // transform in another. (reference: alignment/BH_templateSearch3d_2.m:756-764)
 //
 // Each pass holds a tile of whole columns in LDS and runs a Stockham transform
-// in place: a lane loads the butterflies it owns (at most 18 complex values)
+// in place: a lane loads the butterflies it owns (at most 20 complex values)
 // into registers, the workgroup meets, and they are stored at their sorted
 // places. Per orientation and chunk the passes read and write
 //   z: the template's partial DFT and the tomogram spectrum -> valid z
@@ -388,7 +388,8 @@ static bool col_radices(int n, ColPlan* p) {
 }
 
 // lanes a column: 32 (tiles of 16 columns, 128-byte segments) where the tile
-// fits the LDS of a workgroup, else 64; 0 where neither does
+// fits the LDS of a workgroup, else 64; 0 where neither does: along y and z up to
+// 478 and 903 voxels, along x up to 852 and 1,476 (its columns are half as long)
 static int col_lanes(int n, int table, bool padded) {
   for (int L : {32, 64}) {
     const int W = kColThreads / L;
