@@ -271,8 +271,8 @@ def bench_adjoint(ctx, reps, table="c64"):
 
 def bench_refine(ctx, reps, table="c64", iters=8):
     """The refinement's evaluations: emc_align_refine with eager launches
-    (HIP events per adjoint kernel) over the full support from each
-    particle's start pose."""
+    (HIP events per adjoint kernel, one per run of particles) over the full
+    support from each particle's start pose."""
     for k, (n, count) in enumerate(CLASSES):
         al, starts = _noise_class(ctx, n, count, table, 80 + k)
         al._apply_tuning()
@@ -281,10 +281,10 @@ def bench_refine(ctx, reps, table="c64", iters=8):
         s = DeviceArray.zeros((count, 3), np.float64, ctx)
         wall = _timed(ctx, lambda: al.refine_device(R, s, iters=iters), reps)
         ms, cnt = _ktime(ctx, "align_eval_grad")
-        per = ms / max(cnt, 1)
+        per = ms / (reps * (iters + 1))
         b, samples = eval_grad_bytes(n, count, al.support, table)
         _line("refine", wall, {"kernel": f"cube_eval_kernel<{table}>", "n": n,
-                               "particles": count, "evals_per_call": round(cnt / reps, 2), "kernel_ms": round(per, 4),
+                               "particles": count, "launches_per_call": round(cnt / reps, 2), "kernel_ms": round(per, 4),
                                "bytes": b, "GBps": round(b / (per * 1e-3) / 1e9, 1),
                                "gsamples_per_s": round(samples / (per * 1e-3) / 1e9, 2)})
         del al
@@ -292,8 +292,8 @@ def bench_refine(ctx, reps, table="c64", iters=8):
 
 def bench_search(ctx, reps, table="c64", frac=0.6):
     """The coarse search of a size class: 28 orientations of the 10-degree
-    local grid scored over 0.6 x the support radius (align_pass_kernel +
-    align_final_kernel)."""
+    local grid scored over 0.6 x the support radius (align_pass_kernel, or
+    align_strip_kernel for the fp16 64^3 class, + align_final_kernel)."""
     from .batched import fused_samples_per_unit
     from .geometry import eulerSearch
     grid = eulerSearch("C1", 15, 10, 15, 10)
