@@ -223,3 +223,14 @@ def test_runs_of_particles_within_the_scratch_bound(ctx):
         np.testing.assert_array_equal(c8, cc[q])
         np.testing.assert_array_equal(R8.get(), Rd.get()[q])
         np.testing.assert_array_equal(s8.get(), sd.get()[q])
+
+
+def test_pose_updates_of_more_particles_than_cus(ctx):
+    """Past 256 particles the pose update runs on fewer threads: another order of its
+    FP64 fold and nothing else."""
+    al, R, s = _aligner(12, 260, 5.2, "c64", 12)
+    Rd, sd, cd = al.refine(R, s, iters=2)
+    al.n_part = 8
+    R8, s8, c8 = al.refine(R[:8], s[:8], iters=2)
+    assert np.max(np.abs(Rd[:8] - R8)) < 1e-9 and np.max(np.abs(sd[:8] - s8)) < 1e-9
+    assert np.max(np.abs(cd[:8] - c8)) < 1e-12
